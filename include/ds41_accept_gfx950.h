@@ -44,7 +44,11 @@ int ds41_spark_verify_logits_gpu_v2(const float *target_logits, const float *dra
  * greedy) are unnormalised non-negative fp32 measures; each row is normalised by its fp64
  * mass, with the reference kernel's summation orders, so decisions and tokens equal its.
  * Writes a device ds41_spark_result; an invalid row or draft id gives emitted == -1.
- * One workgroup; no workspace. Returns the launch error (hipErrorInvalidValue for bad
+ * No workspace, no allocation: rows of 2,048 entries or more run on many workgroups over one of 16
+ * scratch slots of the library, claimed and released on the device (calls on several streams may
+ * overlap; with every slot taken a call runs on one workgroup), and *out also carries the slot's
+ * number between the call's launches, so it is not to be read before they have finished. Every row
+ * of p and q is read, also past the step's end. Returns the launch error (hipErrorInvalidValue for bad
  * arguments, as the reference). */
 int ds41_spark_verify_gpu_v2(const int32_t *drafts_dev, const float *q, const float *p,
                              int drafts, int vocab, int greedy, uint64_t seed, uint64_t step,

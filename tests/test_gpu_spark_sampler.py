@@ -56,6 +56,44 @@ def test_verify_gpu_v2_bitexact_vs_oracle(gpu, V, k, kind):
     assert mism == 0
 
 
+@pytest.mark.parametrize("V,k", [(2047, 2), (2048, 2), (2049, 5), (65537, 1), (131072, 2), (131073, 3), (200001, 5)])
+def test_verify_gpu_v2_wide_edges(gpu, V, k):
+    """Around the row length where the call spreads over workgroups, and where a chain of 256 strided
+    or contiguous entries passes one staged block (131,072 entries, 512 per chain)."""
+    rng = np.random.default_rng(V + k)
+    for step, kind in enumerate(("softmax", "sparse", "uniform", "softmax", "sparse", "uniform")):
+        p, q = measures(rng, k + 1, V, kind), measures(rng, k, V, kind)
+        if kind == "softmax":  # close rows: drafts are accepted and later rows reached
+            q = (p[:k] * rng.uniform(0.95, 1.05, (k, V))).astype(np.float32)
+        seed, greedy = int(rng.integers(0, 1 << 63)), int(step == 3)
+        d = (p[:k].argmax(1).astype(np.int32) if greedy
+             else np.array([O.sample_gpu_v2(q[j], seed, step, j, 1) for j in range(k)], np.int32))
+        want = O.verify_gpu_v2(d, q, p, k, V, greedy, seed, step).raw()
+        assert run_gpu(gpu, d, None if greedy else q, p, greedy, seed, step) == want, (kind, greedy)
+
+
+def test_verify_gpu_v2_overlapping_streams(gpu):
+    """Calls in flight on more streams than there are scratch slots, each several times over."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(11)
+    V, k, n = 20000, 3, 24
+    calls = []
+    for i in range(n):
+        p, q = measures(rng, k + 1, V, "softmax"), measures(rng, k, V, "softmax")
+        d = np.array([O.sample_gpu_v2(q[j], i, 5, j, 1) for j in range(k)], np.int32)
+        dev = [torch.from_numpy(a).to(gpu) for a in (d, q, p)]
+        calls.append((dev, torch.zeros((4, 10), dtype=torch.int32, device=gpu), torch.cuda.Stream(),
+                      O.verify_gpu_v2(d, q, p, k, V, 0, i, 5).raw()))
+    torch.cuda.synchronize()
+    for r in range(4):
+        for i, (dev, out, stream, _) in enumerate(calls):
+            G.verify_gpu_v2(*dev, 0, i, 5, out[r], stream)
+    torch.cuda.synchronize()
+    for _, out, _, want in calls:
+        assert all(G.result_raw(out[r]) == want for r in range(4))
+
+
 def test_verify_gpu_v2_invalid_inputs_match_oracle(gpu):
     rng = np.random.default_rng(3)
     V = 5000
