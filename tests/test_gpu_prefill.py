@@ -66,6 +66,29 @@ def test_prefill_raw_vs_oracle(gpu, m, n, k):
     assert np.mean(got == ref) > 0.97
 
 
+@pytest.mark.parametrize("m", [15, 16, 17, 32, 33, 64, 81])
+@pytest.mark.parametrize("n,k,shift", [(136, 224, 0), (130, 256, 8), (257, 288, 3), (127, 1312, 1)])
+def test_prefill_raw_tile_edges(gpu, m, n, k, shift):
+    """Row blocks of 16, 32 and 64; channels past a 128-channel tile; k below, at and past one 256-k slice
+    and in the middle of the third round of slices; weights and scales at any byte offset. Each bf16
+    output rounds a sum of k products once; fp32 sums of up to 41 group dots differ by a few ulp, so at
+    most one output in thirty rounds the other way."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(m * 7 + n + k)
+    w, ws = rand_mx(rng, n, k)
+    xq, xs = O.quantize_mxfp8(rand_x(rng, m, k))
+
+    def at_offset(a):
+        t = torch.zeros(a.size + shift, dtype=torch.uint8, device=gpu)
+        t[shift:] = dev(a.reshape(-1), gpu)
+        return t[shift:].view(a.shape)
+    got = host(G.prefill_raw(at_offset(w), at_offset(ws), dev(xq, gpu), at_offset(xs), m, n, k))
+    _, ref = O.mxfp4_gemm(w, ws, xq, xs, m, n, k)
+    assert rel_l2(O.bf16_to_f32(got), O.bf16_to_f32(ref)) <= 1e-3
+    assert np.mean(got == ref) > 0.97
+
+
 def test_prefill_raw_rejects_like_reference(gpu):
     import ctypes
     import ds41_gfx950 as G
