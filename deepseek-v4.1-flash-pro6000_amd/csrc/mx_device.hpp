@@ -116,11 +116,22 @@ __device__ __forceinline__ bool wait_ready(const ds41_device_expert &e) {
   return false;
 }
 
-__device__ __forceinline__ const uint8_t *proj_weight(const ds41_device_expert &e, int p) {
-  return p == 0 ? e.gate : p == 1 ? e.up : e.down;
+// One projection's weights, scales and residency flag of a table entry, in a caller's registers (a
+// copy of the whole entry, selected between two sources, goes through scratch).
+struct ProjWeights {
+  const uint8_t *w, *s;
+  const uint32_t *ready;
+  uint32_t generation;
+};
+__device__ __forceinline__ ProjWeights proj_weights(const ds41_device_expert &e, int p) {
+  return ProjWeights{p == 0 ? e.gate : p == 1 ? e.up : e.down, p == 0 ? e.gate_scale : p == 1 ? e.up_scale : e.down_scale,
+                     e.ready, e.generation};
 }
-__device__ __forceinline__ const uint8_t *proj_scale(const ds41_device_expert &e, int p) {
-  return p == 0 ? e.gate_scale : p == 1 ? e.up_scale : e.down_scale;
+__device__ __forceinline__ bool wait_ready(const ProjWeights &w) {
+  ds41_device_expert e{};
+  e.ready = w.ready;
+  e.generation = w.generation;
+  return wait_ready(e);
 }
 
 // LDS image of the activation rows of one job: rows of `stride` bytes holding
@@ -593,7 +604,8 @@ __device__ __forceinline__ const uint8_t *weight_row(const uint8_t *w, int row, 
 // byte kb of each dword. Requires U == 8 and k % 1024 == 0 (whole batches).
 // Frees the workgroup's LDS of the weight scales.
 // Tiled: `wrow` from weight_row<true>; pieces are 256 bytes apart.
-template <int U, bool Aligned16, bool GScale = false, bool Tiled = false>
+// AnyAlign: row-major weights at any byte offset.
+template <int U, bool Aligned16, bool GScale = false, bool Tiled = false, bool AnyAlign = false>
 struct Gemv16 {
   const uint8_t *w;  // weight row
   const uint8_t *gs; // GScale: this lane's channel's scale row
@@ -614,6 +626,10 @@ struct Gemv16 {
       return make_uint4(v.x, v.y, v.z, v.w);
     }
     const uint8_t *p = w + 16 * g;
+    if (AnyAlign) {  // one dwordx4 load either way
+      const u32x4 v = *(global_u4u)(p);
+      return make_uint4(v.x, v.y, v.z, v.w);
+    }
     if (Aligned16) {
       const u32x4 v = *(global_u4)(p);
       return make_uint4(v.x, v.y, v.z, v.w);

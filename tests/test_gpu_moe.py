@@ -119,6 +119,66 @@ def test_raw_projection_vs_oracle(gpu, m, n, k):
     assert np.mean(got == ref) > 0.97  # differences are last-place bf16 rounding flips
 
 
+@pytest.mark.parametrize("rows,cols,shift", [(1, 32, 0), (1, 1024, 1), (3, 96, 3), (33, 2880, 0), (1025, 2048, 0)])
+def test_quantize_mxfp8_sizes_bitexact(gpu, rows, cols, shift):
+    """One group, odd group counts, both workgroup sizes (65,536 groups apart), rows at odd offsets."""
+    import ctypes
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(rows + cols)
+    bits = O.bf16_bits((rng.standard_normal((rows, cols)) * rng.choice([1e-6, 1, 3e4], (rows, 1))).astype(np.float32))
+    x = torch.zeros(bits.size + shift, dtype=torch.bfloat16, device=gpu)
+    x[shift:] = dev(bits.reshape(-1), gpu)
+    q = torch.full((bits.size + shift + 1,), 0x55, dtype=torch.uint8, device=gpu)
+    s = torch.full((bits.size // 32 + 1,), 0x55, dtype=torch.uint8, device=gpu)
+    p = ctypes.c_void_p
+    G.check(G.lib().ds41_quantize_mxfp8(p(x[shift:].data_ptr()), p(q[shift:].data_ptr()), p(s.data_ptr()), rows, cols,
+                                        G._stream()), "quantize")
+    qr, sr = O.quantize_mxfp8(bits)
+    assert np.array_equal(host(q)[shift:-1], qr.reshape(-1)) and np.array_equal(host(s)[:-1], sr.reshape(-1))
+    assert host(q)[-1] == 0x55 and host(s)[-1] == 0x55 and (host(q)[:shift] == 0x55).all()  # nothing else written
+
+
+@pytest.mark.parametrize("rows,cols,weighted", [(1, 7, True), (130, 1009, True), (46, 2848, True), (47, 2880, False),
+                                                (46, 2849, True)])
+def test_swiglu_sizes_bitexact(gpu, rows, cols, weighted):
+    """Either side of the eight-element kernel's size (131,072 elements) and columns off its multiple."""
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(rows * cols)
+    g, u = (O.bf16_bits((rng.standard_normal((rows, cols)) * 6).astype(np.float32)) for _ in range(2))
+    w = rng.random(rows).astype(np.float32) if weighted else None
+    got = host(G.swiglu(dev(g, gpu), dev(u, gpu), None if w is None else dev(w, gpu), 10.0))
+    assert np.array_equal(got, O.swiglu(g, u, w, 10.0))
+
+
+@pytest.mark.parametrize("k", [1024, 2048, 992])
+@pytest.mark.parametrize("tokens", [4, 5, 8])
+@pytest.mark.parametrize("p", [0, 2])
+def test_grouped_row_classes(gpu, p, tokens, k):
+    """The row counts either side of the pre-split tile, with scales streamed (k % 1024 == 0) and staged;
+    weights and scales at odd offsets, channels past the last block."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(k + tokens + p)
+    n = 72
+    w, ws = rand_mx(rng, n, k)
+    xq, xs = O.quantize_mxfp8(rand_x(rng, tokens, k))
+
+    def odd(a):
+        t = torch.zeros(a.size + 3, dtype=torch.uint8, device=gpu)
+        t[3:] = dev(a.reshape(-1), gpu)
+        return t[3:]
+    name = ("gate", "up", "down")[p]
+    expert = {name: odd(w), name + "_scale": odd(ws)}  # the table holds bare pointers
+    table, _ = G.device_table([expert], gpu)
+    xd, xsd = dev(xq, gpu), dev(xs, gpu)
+    out = torch.zeros((tokens, n), dtype=torch.bfloat16, device=gpu)
+    G.grouped(table, G.device_jobs([(0, tokens, xd, xsd, out)], gpu), 1, p, n, k)
+    torch.cuda.synchronize()
+    _, ref = O.mxfp4_gemm(w, ws, xq, xs, tokens, n, k)
+    assert rel_l2(O.bf16_to_f32(host(out)), O.bf16_to_f32(ref)) <= 1e-3 and G.take_status() == 0
+
+
 def test_grouped_jobs_all_projections_and_alignment(gpu):
     import torch
     import ds41_gfx950 as G
