@@ -106,45 +106,91 @@ class SparkResult(ctypes.Structure):
                 ("rejected", ctypes.c_int)]
 
 
+# Signatures of every entry point the headers declare, as "result:arguments" with p pointer, s char *,
+# i int, I uint32, Q uint64 / size_t, f float, d double. Declared once, a call converts its arguments in
+# C and takes addresses as plain integers; without them each call built a ctypes object per pointer
+# (six component calls of one small expert: 37 us, 24 us of kernels).
+_SIGNATURES = {
+    "Q:ii": "spark_accept_workspace_bytes spark_sample_workspace_bytes",
+    "i:pppiiddQQppQip": "spark_verify_logits_gpu_v2",
+    "i:pppiiiQQpp": "spark_verify_gpu_v2",
+    "i:piQQIIpp": "spark_sample_gpu_v2",
+    "i:piip": "spark_accept_fallbacks records_extent",
+    "i:piiddQQIIppQip": "spark_sample_logits_gpu_v2",
+    "s:": "spark_error gfx950_version",
+    "i:ppidd": "spark_probabilities",
+    "I:QQIIQ": "spark_rng_word_v2",
+    "d:QQIIQ": "spark_uniform_v2",
+    "i:piQQIIp": "spark_sample_v2",
+    "i:pppiiiQQp": "spark_verify_v2",
+    "i:pppiip": "quantize_mxfp8 quantize_mxfp8_raw dense_quant dequant_mxfp4",
+    "i:ppiiiip": "grouped_mxfp4 grouped_mxfp4_native grouped_mxfp4_parallel grouped_mxfp4_native_parallel "
+                 "grouped_mxfp4_native_tiled xk_grouped_v1",
+    "i:ppppiifp": "swiglu swiglu_raw",
+    "i:ppppiiip": "reduce_experts",
+    "i:pppppiiip": "mxfp4_raw mxfp4_native_raw mxfp4_parallel_raw mxfp4_native_parallel_raw mxfp4_prefill_raw",
+    "i:": "xk_projection_abi_version",
+    "i:ppppiip": "dense_router_scores",
+    "i:pppiiifp": "dense_router_weights",
+    "i:pppip": "engine_route_weights",
+    "i:pppiiip": "router_logits",
+    "i:ppiiip": "router_topk expert_slab_tile",
+    "Q:iiiii": "moe_layer_workspace_bytes moe_prefill_workspace_bytes",
+    "i:pp": "moe_verify_layer moe_verify_layer_noalloc moe_prefill_layer verify_stack_create verify_stack_stats "
+            "pool_policy verify_stack_cache_stats target_experts_create event_record e4m3_converter_check",
+    "Q:": "moe_layer_noalloc_max_bytes",
+    "i:piiiiipi": "moe_layer_plan",
+    "i:ppiiiiip": "grouped_mxfp4_prefill",
+    "i:piiiiip": "moe_prefill_tiles moe_prefill_plan_counts",
+    "i:iip": "expert_slab_layout",
+    "i:ppiii": "expert_slab_tile_host",
+    "i:pppippppp": "verify_stack_step",
+    "i:pippipppp": "verify_stack_layer",
+    "i:p": "verify_stack_destroy host_free pool_destroy pool_reset_history pool_token_release drift_active "
+           "drift_destroy records_free records_count target_experts_destroy take_status",
+    "i:Qp": "host_alloc",
+    "i:pppppiiiip": "dense_fp8",
+    "i:pppppiip": "dense_shared_act",
+    "i:sipppipisQ": "placement_load",
+    "i:iipIIip": "pool_create",
+    "s:p": "pool_error drift_error target_experts_error",
+    "i:ppiip": "pool_acquire",
+    "i:ppip": "pool_borrow spark_topk3_gpu",
+    "i:ppi": "pool_release pool_touch pool_peer pool_switch_target_layer drift_before drift_after",
+    "i:pI": "pool_pin pool_unpin pool_residency pool_decay_interval records_find",
+    "i:pIp": "pool_retain",
+    "i:pipip": "pool_reserve",
+    "i:pi": "pool_drained pool_exclusive pool_fast_minima pool_late events_create events_destroy",
+    "i:ppppsQ": "drift_create",
+    "Q:p": "drift_completed_tokens",
+    "i:pip": "verify_stack_cache records_info",
+    "i:pppi": "verify_stack_prefetch",
+    "i:spsQ": "records_load",
+    "i:psisQ": "records_validate",
+    "i:pipQsQ": "record_read",
+    "i:pipiipQsQ": "record_to_slab",
+    "i:piiipQsQ": "record_load_slab",
+    "i:pippppip": "target_experts",
+    "i:ppp": "event_elapsed_ms",
+    "i:pQpip": "hbm_read_probe",
+    "i:pQpiiip": "hbm_read_probe_ex",
+}
+_CTYPES = {"p": ctypes.c_void_p, "s": ctypes.c_char_p, "i": ctypes.c_int, "I": ctypes.c_uint32, "Q": ctypes.c_uint64,
+           "f": ctypes.c_float, "d": ctypes.c_double}
+
+
 def lib():
     global _lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(f"{LIB_PATH} is not built: run __graft_entry__.build()")
-        _lib = ctypes.CDLL(LIB_PATH)
-        _lib.ds41_moe_layer_workspace_bytes.restype = ctypes.c_size_t
-        _lib.ds41_moe_layer_noalloc_max_bytes.restype = ctypes.c_size_t
-        _lib.ds41_drift_completed_tokens.restype = ctypes.c_uint64
-        _lib.ds41_drift_error.restype = ctypes.c_char_p
-        _lib.ds41_moe_prefill_workspace_bytes.restype = ctypes.c_size_t
-        _lib.ds41_gfx950_version.restype = ctypes.c_char_p
-        _lib.ds41_spark_accept_workspace_bytes.restype = ctypes.c_size_t
-        _lib.ds41_spark_sample_workspace_bytes.restype = ctypes.c_size_t
-        _lib.ds41_spark_sample_logits_gpu_v2.argtypes = [
-            ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_uint64,
-            ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
-            ctypes.c_int, ctypes.c_void_p]
-        _lib.ds41_spark_error.restype = ctypes.c_char_p
-        _lib.ds41_spark_rng_word_v2.restype = ctypes.c_uint32
-        _lib.ds41_spark_uniform_v2.restype = ctypes.c_double
-        _lib.ds41_spark_verify_gpu_v2.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
-                                                  ctypes.c_int, ctypes.c_int, ctypes.c_uint64, ctypes.c_uint64,
-                                                  ctypes.c_void_p, ctypes.c_void_p]
-        _lib.ds41_spark_sample_gpu_v2.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_uint64, ctypes.c_uint64,
-                                                  ctypes.c_uint32, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_void_p]
-        _lib.ds41_pool_error.restype = ctypes.c_char_p
-        _lib.ds41_pool_error.argtypes = [ctypes.c_void_p]
-        _lib.ds41_placement_load.argtypes = [ctypes.c_char_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
-                                             ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
-                                             ctypes.c_char_p, ctypes.c_size_t]
-        _lib.ds41_target_experts_error.restype = ctypes.c_char_p
-        _lib.ds41_target_experts_error.argtypes = [ctypes.c_void_p]
-        _lib.ds41_target_experts.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
-                                             ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
-        _lib.ds41_spark_verify_logits_gpu_v2.argtypes = [
-            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_double,
-            ctypes.c_double, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
-            ctypes.c_int, ctypes.c_void_p]
+        L = ctypes.CDLL(LIB_PATH)
+        for sig, names in _SIGNATURES.items():
+            ret, args = sig.split(":")
+            for name in names.split():
+                f = getattr(L, "ds41_" + name)
+                f.restype, f.argtypes = _CTYPES[ret], [_CTYPES[a] for a in args]
+        _lib = L
     return _lib
 
 
@@ -154,13 +200,24 @@ def check(rc, what):
 
 
 def _p(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    """Address of a tensor (None: null), as every declared entry point takes it."""
+    return None if t is None else t.data_ptr()
+
+
+_torch = None
 
 
 def _stream(stream=None):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    """hipStream_t of a torch stream, or of the current one."""
+    if stream is not None:
+        return stream.cuda_stream
+    global _torch
+    if _torch is None:
+        import torch
+        _torch = torch
+    if _torch.cuda.is_initialized():  # the handle itself, without building a Stream object
+        return _torch._C._cuda_getCurrentRawStream(_torch._C._cuda_getDevice())
+    return _torch.cuda.current_stream().cuda_stream
 
 
 def take_status():
@@ -290,18 +347,13 @@ def router_weights(u, ids, scale=1.5, stream=None):
 def hbm_read_probe(buf, sink, blocks, stream=None):
     """Streams buf (a uint8 CUDA tensor, 16-byte multiple) once with `blocks` workgroups; sink
     holds blocks * 256 uint32 words. Time it to get the device's streaming-read ceiling."""
-    f = lib().ds41_hbm_read_probe
-    f.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
-    check(f(buf.data_ptr(), buf.numel(), sink.data_ptr(), blocks, _stream(stream)), "ds41_hbm_read_probe")
+    check(lib().ds41_hbm_read_probe(buf.data_ptr(), buf.numel(), sink.data_ptr(), blocks, _stream(stream)), "ds41_hbm_read_probe")
 
 
 def hbm_read_probe_ex(buf, sink, blocks, loads_in_flight, nontemporal, stream=None):
     """hbm_read_probe with loads_in_flight (4, 8, 16) 16-byte loads per thread in flight, plain or
     non-temporal loads."""
-    f = lib().ds41_hbm_read_probe_ex
-    f.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                  ctypes.c_void_p]
-    check(f(buf.data_ptr(), buf.numel(), sink.data_ptr(), blocks, loads_in_flight, int(nontemporal),
+    check(lib().ds41_hbm_read_probe_ex(buf.data_ptr(), buf.numel(), sink.data_ptr(), blocks, loads_in_flight, int(nontemporal),
             _stream(stream)), "ds41_hbm_read_probe_ex")
 
 
@@ -419,7 +471,7 @@ def verify_logits(target, draft, drafts_dev, temperature, top_p, seed, step, out
     check(lib().ds41_spark_verify_logits_gpu_v2(
         target.data_ptr(), 0 if draft is None else draft.data_ptr(), 0 if k == 0 else drafts_dev.data_ptr(), k, V,
         float(temperature), float(top_p), seed, step, out.data_ptr(), workspace.data_ptr(), workspace.numel(),
-        flags, _stream(stream).value), "ds41_spark_verify_logits_gpu_v2")
+        flags, _stream(stream)), "ds41_spark_verify_logits_gpu_v2")
 
 
 def sample_workspace(rows, vocab, device="cuda"):
@@ -433,7 +485,7 @@ def sample_logits_rc(logits, temperature, top_p, seed, step, first_slot, purpose
     rows, V = logits.shape
     return lib().ds41_spark_sample_logits_gpu_v2(
         logits.data_ptr(), rows, V, float(temperature), float(top_p), seed, step, first_slot, purpose,
-        tokens.data_ptr(), workspace.data_ptr(), workspace.numel(), flags, _stream(stream).value)
+        tokens.data_ptr(), workspace.data_ptr(), workspace.numel(), flags, _stream(stream))
 
 
 def sample_logits(logits, temperature, top_p, seed, step, first_slot, purpose, tokens, workspace, flags=0,

@@ -34,6 +34,32 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
 
 
+def test_binding_declares_every_entry_point():
+    """The binding passes device addresses as plain integers, so each entry point needs its argument types:
+    every declared function is listed once, with the header's result and argument kinds."""
+    import sys
+    sys.path.insert(0, os.path.join(ROOT, "deepseek-v4.1-flash-pro6000_amd"))
+    import ds41_gfx950 as G
+
+    def kind(a):
+        a = a.strip()
+        if "*" in a or "[" in a:
+            return "s" if "char" in a else "p"
+        for t, k in (("uint64_t", "Q"), ("size_t", "Q"), ("uint32_t", "I"), ("double", "d"), ("float", "f"), ("int", "i")):
+            if t in a:
+                return k
+        return ""
+    want = {}
+    for h in glob.glob(os.path.join(ROOT, "include", "*.h")):
+        text = re.sub(r"/\*.*?\*/", "", open(h).read(), flags=re.S)
+        for m in re.finditer(r"^([A-Za-z_][\w\s\*]*?)\b(ds41_\w+)\s*\(([^;{]*)\)\s*;", text, flags=re.M):
+            args = " ".join(m.group(3).split())
+            want[m.group(2)] = kind(m.group(1)) + ":" + "".join(kind(a) for a in args.split(","))
+    listed = [("ds41_" + n, sig) for sig, names in G._SIGNATURES.items() for n in names.split()]
+    assert len(listed) == len(dict(listed)) and dict(listed) == want and set(want) == declared()
+    assert all(getattr(G.lib(), n).argtypes is not None for n in want)
+
+
 def test_abi_struct_sizes():
     import sys
     sys.path.insert(0, os.path.join(ROOT, "deepseek-v4.1-flash-pro6000_amd"))
