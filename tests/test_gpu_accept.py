@@ -260,3 +260,26 @@ def test_accept_top_p_cluster_of_adjacent_logits(gpu, cluster):
     got, want, _ = bonus_draws(gpu, x, 1.0, 0.5, 24)
     assert got == want
     assert all(100 <= t[0] < 100 + cluster for t in got)
+
+
+@pytest.mark.parametrize("top_p", [1.0, 0.9])
+@pytest.mark.parametrize("V", [1, 63, 2047, 2049, 131072, 131073, 262145])
+def test_accept_row_edges_vs_oracle(gpu, V, top_p):
+    """Row lengths at the edges of the kernels' splits: one element, one chunk less and more an element,
+    64 and 65 chunks of 2,048 (the statistics' wave holds one chunk a lane, then more), a workgroup's
+    share of 4,096 elements (32 workgroups x 4,096 = 131,072) in one block and in several. The steps'
+    results are the oracle's."""
+    import torch
+    import ds41_gfx950 as G
+    k = 2
+    ws = G.accept_workspace(k, V, gpu)
+    out = torch.zeros(16, dtype=torch.int32, device=gpu)
+    rng = np.random.default_rng(V)
+    for step in range(6):
+        target, draft = sweep_logits(rng, k, V, 2.5, 0.5, "rounded" if step & 1 else "normal")
+        q = [O.probabilities(draft[j], 1.0, top_p) for j in range(k)]
+        drafts = np.array([O.sample_v2(q[j], 11, step, j, 1) for j in range(k)], np.int32)
+        G.verify_logits(torch.from_numpy(target).to(gpu), torch.from_numpy(draft).to(gpu),
+                        torch.from_numpy(drafts).to(gpu), 1.0, top_p, 11, step, out, ws)
+        torch.cuda.synchronize()
+        assert G.result_tuple(out) == oracle_tuple(target, draft, drafts, 1.0, top_p, 11, step), step
