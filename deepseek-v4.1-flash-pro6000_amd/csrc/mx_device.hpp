@@ -604,42 +604,54 @@ __device__ __forceinline__ const uint8_t *weight_row(const uint8_t *w, int row, 
 // byte kb of each dword. Requires U == 8 and k % 1024 == 0 (whole batches).
 // Frees the workgroup's LDS of the weight scales.
 // Tiled: `wrow` from weight_row<true>; pieces are 256 bytes apart.
-// AnyAlign: row-major weights at any byte offset.
-template <int U, bool Aligned16, bool GScale = false, bool Tiled = false, bool AnyAlign = false>
+// Row-major weights may lie at any byte offset.
+template <int U, bool GScale = false, bool Tiled = false, bool FreeOrder = false>
 struct Gemv16 {
-  const uint8_t *w;  // weight row
+  static_assert(U % 2 == 0, "chunks are loaded in pairs");
+  const uint8_t *w;  // weight row (row-major: row l & 7 of the wave's 16)
+  int d8;            // row-major: offset of row 8 + (l & 7)
   const uint8_t *gs; // GScale: this lane's channel's scale row
   int kb, ng, nch, nb;
   uint4 A[U], B[U];
   uint4 SA[2], SB[2];
 
-  // 16 bytes of K32 group min(4c + kb, ng - 1) through a global-address-space
-  // pointer (global_load, counted by vmcnt only, never by lgkmcnt). Plain (not
-  // non-temporal) loads: each 128-byte row line is consumed by two consecutive
-  // chunk loads, and the second one must still find the line in L2.
-  __device__ __forceinline__ uint4 ld(int c) const {
+  // 16 bytes of K32 group min(4c + kb, ng - 1) of the row at `row`, through a
+  // global-address-space pointer (global_load, counted by vmcnt only, never by lgkmcnt).
+  __device__ __forceinline__ uint4 ld(const uint8_t *row, int c) const {
     const int cc = c < nch ? c : nch - 1;
     int g = 4 * cc + kb;
     g = g < ng ? g : ng - 1;
     if (Tiled) {  // each kilobyte block is read by this one instruction: no reuse to keep in the caches
-      const u32x4 v = __builtin_nontemporal_load((global_u4)(w + 256 * g));
+      const u32x4 v = __builtin_nontemporal_load((global_u4)(row + 256 * g));
       return make_uint4(v.x, v.y, v.z, v.w);
     }
-    const uint8_t *p = w + 16 * g;
-    if (AnyAlign) {  // one dwordx4 load either way
-      const u32x4 v = *(global_u4u)(p);
-      return make_uint4(v.x, v.y, v.z, v.w);
-    }
-    if (Aligned16) {
-      const u32x4 v = *(global_u4)(p);
-      return make_uint4(v.x, v.y, v.z, v.w);
-    }
-    const u32x2 lo = *(global_u2)(p), hi = *(global_u2)(p + 8);
-    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    const u32x4 v = __builtin_nontemporal_load((global_u4u)(row + 16 * g));  // any alignment: one dwordx4
+    return make_uint4(v.x, v.y, v.z, v.w);
   }
+  // Row-major: a chunk is 64 bytes of a row, half a cache line, and a load of one chunk of 16 rows
+  // would touch 16 lines for half of each. So a pair of chunks is loaded as two instructions of 8 whole
+  // lines each (rows 0..7, then 8..15; the upper 8 lanes of each 16 take the second chunk), and
+  // pair_chunks() hands each lane its own row's pieces. Every line is then read by one instruction, so
+  // the loads are non-temporal as the tiled layout's are. A layer of 8 rows (hidden 4,096, 49 experts of
+  // 2,880 channels) goes from 184 to 172 us, 23 jobs on experts of that size from 106 to 100 us; without
+  // the non-temporal loads the layer stayed at 182 us.
   __device__ __forceinline__ void load(uint4 *buf, int b) const {
 #pragma unroll
-    for (int u = 0; u < U; ++u) buf[u] = ld(b * U + u);
+    for (int u = 0; u < U; ++u)
+      buf[u] = Tiled ? ld(w, b * U + u) : ld(u & 1 ? w + d8 : w, b * U + (u & ~1) + ((int)(threadIdx.x >> 3) & 1));
+  }
+  // Chunks u and u + 1 of the lane's own row from a loaded pair: lane l < 8 (of 16) holds its row's
+  // chunk u in x0 and its chunk u + 1 is in lane l + 8's x0; lane l >= 8 holds its chunk u + 1 in x1
+  // and its chunk u is in lane l - 8's x1 (row_ror 8 is the swap of the two halves of 16 lanes).
+  __device__ __forceinline__ static uint32_t half_swap(uint32_t own, uint32_t other, bool upper) {
+    return upper ? (uint32_t)__builtin_amdgcn_update_dpp((int)own, (int)other, 0x128, 0xf, 0xc, false)
+                 : (uint32_t)__builtin_amdgcn_update_dpp((int)own, (int)other, 0x128, 0xf, 0x3, false);
+  }
+  __device__ __forceinline__ static void pair_chunks(uint4 x0, uint4 x1, uint4 &c0, uint4 &c1) {
+    c0 = make_uint4(half_swap(x0.x, x1.x, true), half_swap(x0.y, x1.y, true), half_swap(x0.z, x1.z, true),
+                    half_swap(x0.w, x1.w, true));
+    c1 = make_uint4(half_swap(x1.x, x0.x, false), half_swap(x1.y, x0.y, false), half_swap(x1.z, x0.z, false),
+                    half_swap(x1.w, x0.w, false));
   }
   __device__ __forceinline__ void ld_scales(uint4 *S, int b) const {
     // any alignment: gfx950 global loads take unaligned addresses (one dwordx4 either way)
@@ -657,6 +669,15 @@ struct Gemv16 {
   __device__ __forceinline__ void begin(const uint8_t *wrow, int k, const uint8_t *gscale_row = nullptr) {
     kb = (threadIdx.x & 63) >> 4;
     w = wrow;
+    d8 = 0;
+    if (!Tiled) {  // the rows of the lane and of the lane 8 apart
+      const uint64_t a = (uint64_t)wrow;
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)a, 0x128, 0xf, 0xf, false),
+                     hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(a >> 32), 0x128, 0xf, 0xf, false);
+      const uint8_t *o = (const uint8_t *)(((uint64_t)hi << 32) | lo);
+      d8 = (int)(threadIdx.x & 8 ? wrow - o : o - wrow);
+      if (threadIdx.x & 8) w = o;
+    }
     gs = gscale_row;
     ng = k >> 5;
     nch = (ng + 3) >> 2;
@@ -685,10 +706,11 @@ struct Gemv16 {
       const v8i bv = v8i{(int)wv.x, (int)wv.y, (int)wv.z, (int)wv.w, 0, 0, 0, 0};
       acc = mfma_chunk(lo, hi, bv, acc, (int)sa[4 * cx], sw);
     };
-    auto compute = [&](const uint4 *buf, const uint4 *S, int b) {
+    auto compute = [&](uint4 *buf, const uint4 *S, int b) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int c = b * U + u;
+        if (!Tiled && !(u & 1)) pair_chunks(buf[u], buf[u + 1], buf[u], buf[u + 1]);
         int sw;
         if (GScale) {  // byte kb of dword u of the batch's scale window
           const uint4 &w4 = S[u >> 2];
@@ -700,6 +722,10 @@ struct Gemv16 {
           sw = (int)lsw[g];
         }
         mma(buf[u], c, sw);
+        // Pair by pair: without the fence the swaps of the whole batch are hoisted, which took the layer's
+        // row-major gate/up from 124 to 148 VGPRs, from four waves a SIMD to three (182 -> 191 us). A
+        // pre-split tile with FreeOrder has the registers and is 1 % faster without it.
+        if (!Tiled && (Split || !FreeOrder) && (u & 1)) __builtin_amdgcn_sched_barrier(0);
       }
     };
     int b = 0;

@@ -179,6 +179,27 @@ def test_grouped_row_classes(gpu, p, tokens, k):
     assert rel_l2(O.bf16_to_f32(host(out)), O.bf16_to_f32(ref)) <= 1e-3 and G.take_status() == 0
 
 
+@pytest.mark.parametrize("k", [32, 128, 160, 384, 1056])
+def test_grouped_odd_chunk_pairs(gpu, k):
+    """Row-major weights are streamed in pairs of 128-element chunks: a pair with no, part of or all of its
+    second chunk inside the row, rows at an odd byte offset and a last block of 8 channels."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(k)
+    n, tokens = 72, 3
+    w, ws = rand_mx(rng, n, k)
+    xq, xs = O.quantize_mxfp8(rand_x(rng, tokens, k))
+    buf = torch.zeros(w.size + 5, dtype=torch.uint8, device=gpu)
+    buf[5:] = dev(w.reshape(-1), gpu)
+    sd, xd, xsd = dev(ws, gpu), dev(xq, gpu), dev(xs, gpu)
+    table, _ = G.device_table([{"up": buf[5:], "up_scale": sd}], gpu)
+    out = torch.zeros((tokens, n), dtype=torch.bfloat16, device=gpu)
+    G.grouped(table, G.device_jobs([(0, tokens, xd, xsd, out)], gpu), 1, 1, n, k)
+    torch.cuda.synchronize()
+    _, ref = O.mxfp4_gemm(w, ws, xq, xs, tokens, n, k)
+    assert rel_l2(O.bf16_to_f32(host(out)), O.bf16_to_f32(ref)) <= 1e-3 and G.take_status() == 0
+
+
 def test_grouped_jobs_all_projections_and_alignment(gpu):
     import torch
     import ds41_gfx950 as G
