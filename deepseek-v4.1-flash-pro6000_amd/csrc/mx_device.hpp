@@ -634,8 +634,9 @@ __device__ __forceinline__ const uint8_t *weight_row(const uint8_t *w, int row, 
 // byte kb of each dword. Requires U == 8 and k % 1024 == 0 (whole batches).
 // Frees the workgroup's LDS of the weight scales.
 // Tiled: `wrow` from weight_row<true>; pieces are 256 bytes apart.
-// Row-major weights may lie at any byte offset.
-template <int U, bool GScale = false, bool Tiled = false, bool FreeOrder = false>
+// Row-major weights may lie at any byte offset. Once: non-temporal loads (a row that is not whole
+// 128-byte lines long leaves parts of lines to the next load of the row, and may want them cached).
+template <int U, bool GScale = false, bool Tiled = false, bool FreeOrder = false, bool Once = true>
 struct Gemv16 {
   static_assert(U % 2 == 0, "chunks are loaded in pairs");
   const uint8_t *w;  // weight row (row-major: row l & 7 of the wave's 16)
@@ -655,7 +656,8 @@ struct Gemv16 {
       const u32x4 v = __builtin_nontemporal_load((global_u4)(row + 256 * g));
       return make_uint4(v.x, v.y, v.z, v.w);
     }
-    const u32x4 v = __builtin_nontemporal_load((global_u4u)(row + 16 * g));  // any alignment: one dwordx4
+    const global_u4u p = (global_u4u)(row + 16 * g);  // any alignment: one dwordx4
+    const u32x4 v = Once ? __builtin_nontemporal_load(p) : *p;
     return make_uint4(v.x, v.y, v.z, v.w);
   }
   // Row-major: a chunk is 64 bytes of a row, half a cache line, and a load of one chunk of 16 rows
