@@ -89,6 +89,14 @@ def test_tiled_layer_bitexact(gpu, T, H, I, E, K, shared, fp8):
             assert diff == 0 and not np.any(out[1][0] == 0x7fc0)
 
 
+@pytest.mark.parametrize("I", [2304, 2880])
+def test_tiled_layer_bitexact_down_rows(gpu, I):
+    """Row-major down rows of whole 128-byte lines (I = 2,304) and not (2,880) take different loads in the
+    separate down kernel (T = 8, K = 8); both give the tiled layout's bits."""
+    test_tiled_layer_bitexact(gpu, 8, 1024, I, 64, 8, True, False)
+
+
+
 def test_tiled_stack_with_host_tier_and_cache_bitexact(gpu):
     """A 3-layer stack at configs[4]'s layer shape (16 host-tier experts per layer) in both layouts: the tiled
     stack's host slabs are tiled too. Router routing and Zipf-like given ids; then both stacks get an HBM cache
