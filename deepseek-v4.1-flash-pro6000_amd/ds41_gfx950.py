@@ -115,6 +115,7 @@ _SIGNATURES = {
     "i:pppiiddQQppQip": "spark_verify_logits_gpu_v2",
     "i:pppiiiQQpp": "spark_verify_gpu_v2",
     "i:piQQIIpp": "spark_sample_gpu_v2",
+    "i:ipp": "spark_scratch_hold",
     "i:piip": "spark_accept_fallbacks records_extent",
     "i:piiddQQIIppQip": "spark_sample_logits_gpu_v2",
     "s:": "spark_error gfx950_version",
@@ -565,6 +566,12 @@ def verify_gpu_v2(drafts_dev, q, p, greedy, seed, step, out, stream=None):
 def sample_gpu_v2(p, seed, step, slot, purpose, out, stream=None):
     check(lib().ds41_spark_sample_gpu_v2(_p(p), p.shape[0], seed, step, slot, purpose, _p(out), _stream(stream)),
           "ds41_spark_sample_gpu_v2")
+
+
+def spark_scratch_hold(hold, in_use, stream=None):
+    """Testing: hold takes the samplers' free scratch slots, not hold gives them back; in_use (device int32)
+    gets the number of slots that calls own."""
+    check(lib().ds41_spark_scratch_hold(int(hold), _p(in_use), _stream(stream)), "ds41_spark_scratch_hold")
 
 
 def result_raw(buf):

@@ -46,17 +46,20 @@ int ds41_spark_verify_logits_gpu_v2(const float *target_logits, const float *dra
  * Writes a device ds41_spark_result; an invalid row or draft id gives emitted == -1.
  * No workspace, no allocation: rows of 2,048 entries or more run on many workgroups over one of 16
  * scratch slots of the library, claimed and released on the device (calls on several streams may
- * overlap; with every slot taken a call runs on one workgroup), and *out also carries the slot's
- * number between the call's launches, so it is not to be read before they have finished. Every row
- * of p and q is read, also past the step's end. Returns the launch error (hipErrorInvalidValue for bad
- * arguments, as the reference). */
+ * overlap; with every slot taken a call runs on one workgroup). *out is written once, by the call's
+ * last launch, so the drafts may lie inside it. Every row of p and q is read, also past the step's
+ * end. Returns the launch error (hipErrorInvalidValue for bad arguments, as the reference). */
 int ds41_spark_verify_gpu_v2(const int32_t *drafts_dev, const float *q, const float *p,
                              int drafts, int vocab, int greedy, uint64_t seed, uint64_t step,
                              ds41_spark_result *out, void *stream);
 /* sample_kernel (sampling.cu:23,48): one token of measure p with the v2 uniform of
- * (seed, step, slot, purpose); -1 for an invalid row. out: device int32. */
+ * (seed, step, slot, purpose); -1 for an invalid row. out: device int32, written once, by the
+ * call's last launch (the scratch slots of ds41_spark_verify_gpu_v2). */
 int ds41_spark_sample_gpu_v2(const float *p, int vocab, uint64_t seed, uint64_t step, uint32_t slot,
                              uint32_t purpose, int32_t *out, void *stream);
+/* Testing: hold != 0 takes every free scratch slot of the two entries above on the current device, so
+ * that calls find none; 0 gives those back. *in_use (device): the slots that calls in flight own. */
+int ds41_spark_scratch_hold(int hold, int32_t *in_use, void *stream);
 /* Number of accept steps that took the sequential path since the workspace was
  * zeroed (synchronous read). */
 int ds41_spark_accept_fallbacks(const void *workspace, int drafts, int vocab, uint32_t *count);

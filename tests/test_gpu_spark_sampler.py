@@ -72,8 +72,121 @@ def test_verify_gpu_v2_wide_edges(gpu, V, k):
         assert run_gpu(gpu, d, None if greedy else q, p, greedy, seed, step) == want, (kind, greedy)
 
 
+def slots_in_use(gpu, hold=0):
+    """Scratch slots that calls own; hold: takes the free ones first."""
+    import torch
+    import ds41_gfx950 as G
+    n = torch.full((1,), -1, dtype=torch.int32, device=gpu)
+    G.spark_scratch_hold(hold, n)
+    torch.cuda.synchronize()
+    return int(n.item())
+
+
+def accepting_call(gpu, rng, V, k, seed, step):
+    """A call whose rows are close, so that drafts are accepted: its arrays, and the same on the device."""
+    import torch
+    p = measures(rng, k + 1, V, "softmax")
+    q = (p[:k] * rng.uniform(0.95, 1.05, (k, V))).astype(np.float32)
+    d = np.array([O.sample_gpu_v2(q[j], seed, step, j, 1) for j in range(k)], np.int32)
+    return (d, q, p), [torch.from_numpy(a).to(gpu) for a in (d, q, p)]
+
+
+@pytest.mark.parametrize("V", [1000, 20000])
+def test_verify_gpu_v2_drafts_inside_result(gpu, V):
+    """The drafts lie in the result's own tokens: both ways of running a call read them before it is written."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(V)
+    k = 3
+    for step in range(6):
+        (d, q, p), (_, qd, pd) = accepting_call(gpu, rng, V, k, 9, step)
+        for greedy in (0, 1):
+            if greedy:
+                d = p[:k].argmax(1).astype(np.int32)
+            out = torch.full((10,), 7, dtype=torch.int32, device=gpu)
+            out[:k] = torch.from_numpy(d).to(gpu)
+            G.verify_gpu_v2(out[:k], None if greedy else qd, pd, greedy, 9, step, out)
+            torch.cuda.synchronize()
+            assert G.result_raw(out) == O.verify_gpu_v2(d, None if greedy else q, p, k, V, greedy, 9, step).raw()
+
+
+def test_wide_calls_with_one_result_buffer(gpu):
+    """The same call on several streams into one result: whatever order the launches take, each finds its own
+    slot, the result is the call's, and every slot is free in the end."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(12)
+    V, k = 20000, 3
+    host, dev = accepting_call(gpu, rng, V, k, 3, 4)
+    want = O.verify_gpu_v2(*host, k, V, 0, 3, 4).raw()
+    out, tok = torch.zeros(10, dtype=torch.int32, device=gpu), torch.zeros(1, dtype=torch.int32, device=gpu)
+    streams = [torch.cuda.Stream() for _ in range(8)]
+    torch.cuda.synchronize()
+    for r in range(12):
+        for s in streams:
+            G.verify_gpu_v2(*dev, 0, 3, 4, out, s)
+            G.sample_gpu_v2(dev[2][0], 3, 4, 0, 0, tok, s)
+    torch.cuda.synchronize()
+    assert G.result_raw(out) == want
+    assert int(tok.item()) == O.sample_gpu_v2(host[2][0], 3, 4, 0, 0)
+    assert slots_in_use(gpu) == 0
+
+
+def test_wide_calls_without_a_free_slot(gpu):
+    """With every slot taken, verify (greedy and not) and sample run on one workgroup, with the same results."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(13)
+    V, k = 20000, 3
+    host, dev = accepting_call(gpu, rng, V, k, 5, 6)
+    top = host[2][:k].argmax(1).astype(np.int32)
+    topd = torch.from_numpy(top).to(gpu)
+    outs = [torch.zeros(10, dtype=torch.int32, device=gpu) for _ in range(4)]
+    toks = [torch.zeros(1, dtype=torch.int32, device=gpu) for _ in range(2)]
+    try:
+        for i in range(2):  # all taken, then all free
+            assert slots_in_use(gpu, hold=1 - i) == 0
+            G.verify_gpu_v2(*dev, 0, 5, 6, outs[2 * i])
+            G.verify_gpu_v2(topd, None, dev[2], 1, 5, 6, outs[2 * i + 1])
+            G.sample_gpu_v2(dev[2][1], 5, 6, 1, 0, toks[i])
+            torch.cuda.synchronize()
+    finally:
+        slots_in_use(gpu, hold=0)
+    for i in range(2):
+        assert G.result_raw(outs[2 * i]) == O.verify_gpu_v2(*host, k, V, 0, 5, 6).raw()
+        assert G.result_raw(outs[2 * i + 1]) == O.verify_gpu_v2(top, None, host[2], k, V, 1, 5, 6).raw()
+        assert int(toks[i].item()) == O.sample_gpu_v2(host[2][1], 5, 6, 1, 0)
+    assert slots_in_use(gpu) == 0
+
+
+def test_wide_call_replayed(gpu):
+    """A captured call finds its slot again at every replay, with eager calls between and new inputs in place."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(14)
+    V, k = 20000, 2
+    _, dev = accepting_call(gpu, rng, V, k, 7, 8)
+    out, eager = (torch.zeros(10, dtype=torch.int32, device=gpu) for _ in range(2))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        G.verify_gpu_v2(*dev, 0, 7, 8, out, stream)
+    for _ in range(4):
+        host, new = accepting_call(gpu, rng, V, k, 7, 8)
+        for a, b in zip(dev, new):
+            a.copy_(b)
+        torch.cuda.synchronize()
+        G.verify_gpu_v2(*dev, 0, 7, 8, eager)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert G.result_raw(out) == G.result_raw(eager) == O.verify_gpu_v2(*host, k, V, 0, 7, 8).raw()
+    assert slots_in_use(gpu) == 0
+
+
 def test_verify_gpu_v2_overlapping_streams(gpu):
-    """Calls in flight on more streams than there are scratch slots, each several times over."""
+    """Calls on more streams than there are scratch slots, each several times over; every slot is free again
+    in the end (the hardware's queues decide how many of them are in flight together)."""
     import torch
     import ds41_gfx950 as G
     rng = np.random.default_rng(11)
@@ -92,6 +205,7 @@ def test_verify_gpu_v2_overlapping_streams(gpu):
     torch.cuda.synchronize()
     for _, out, _, want in calls:
         assert all(G.result_raw(out[r]) == want for r in range(4))
+    assert slots_in_use(gpu) == 0
 
 
 def test_verify_gpu_v2_invalid_inputs_match_oracle(gpu):
