@@ -44,7 +44,7 @@ int ds41_spark_verify_logits_gpu_v2(const float *target_logits, const float *dra
  * greedy) are unnormalised non-negative fp32 measures; each row is normalised by its fp64
  * mass, with the reference kernel's summation orders, so decisions and tokens equal its.
  * Writes a device ds41_spark_result; an invalid row or draft id gives emitted == -1.
- * No workspace, no allocation: rows of 2,048 entries or more run on many workgroups over one of 16
+ * No workspace, no allocation: long rows (4,096 to 10,240 entries or more) run on many workgroups over one of 16
  * scratch slots of the library, claimed and released on the device (calls on several streams may
  * overlap; with every slot taken a call runs on one workgroup). *out is written once, by the call's
  * last launch, so the drafts may lie inside it. Every row of p and q is read, also past the step's

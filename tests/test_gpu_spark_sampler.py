@@ -56,9 +56,10 @@ def test_verify_gpu_v2_bitexact_vs_oracle(gpu, V, k, kind):
     assert mism == 0
 
 
-@pytest.mark.parametrize("V,k", [(2047, 2), (2048, 2), (2049, 5), (65537, 1), (131072, 2), (131073, 3), (200001, 5)])
+@pytest.mark.parametrize("V,k", [(2047, 2), (2048, 2), (2049, 5), (4095, 2), (4096, 2), (4097, 5), (5119, 1), (5120, 1), (5121, 4),
+                                 (65537, 1), (131072, 2), (131073, 3), (200001, 5)])
 def test_verify_gpu_v2_wide_edges(gpu, V, k):
-    """Around the row length where the call spreads over workgroups, and where a chain of 256 strided
+    """Around the row lengths where calls spread over workgroups, and where a chain of 256 strided
     or contiguous entries passes one staged block (131,072 entries, 512 per chain)."""
     rng = np.random.default_rng(V + k)
     for step, kind in enumerate(("softmax", "sparse", "uniform", "softmax", "sparse", "uniform")):
@@ -70,6 +71,23 @@ def test_verify_gpu_v2_wide_edges(gpu, V, k):
              else np.array([O.sample_gpu_v2(q[j], seed, step, j, 1) for j in range(k)], np.int32))
         want = O.verify_gpu_v2(d, q, p, k, V, greedy, seed, step).raw()
         assert run_gpu(gpu, d, None if greedy else q, p, greedy, seed, step) == want, (kind, greedy)
+
+
+@pytest.mark.parametrize("V", [10239, 10240, 10241])
+def test_single_row_wide_edges(gpu, V):
+    """The row length from which a call of one row spreads over workgroups: sample, and verify of no draft."""
+    import torch
+    import ds41_gfx950 as G
+    rng = np.random.default_rng(V)
+    tok = torch.zeros(1, dtype=torch.int32, device=gpu)
+    for step, kind in enumerate(("softmax", "sparse", "uniform")):
+        p = measures(rng, 1, V, kind)
+        for greedy in (0, 1):
+            want = O.verify_gpu_v2(None, None, p, 0, V, greedy, 21, step).raw()
+            assert run_gpu(gpu, None, None, p, greedy, 21, step) == want, (kind, greedy)
+        G.sample_gpu_v2(torch.from_numpy(p[0]).to(gpu), 21, step, 2, 1, tok)
+        torch.cuda.synchronize()
+        assert int(tok.item()) == O.sample_gpu_v2(p[0], 21, step, 2, 1), kind
 
 
 def slots_in_use(gpu, hold=0):
