@@ -140,9 +140,11 @@ def test_quantize_mxfp8_sizes_bitexact(gpu, rows, cols, shift):
 
 
 @pytest.mark.parametrize("rows,cols,weighted", [(1, 7, True), (130, 1009, True), (46, 2848, True), (47, 2880, False),
-                                                (46, 2849, True)])
+                                                (46, 2849, True), (47, 2880, True), (455, 2880, True), (456, 2880, True),
+                                                (456, 2880, False), (457, 2869, True), (163840, 8, True), (936, 2880, True)])
 def test_swiglu_sizes_bitexact(gpu, rows, cols, weighted):
-    """Either side of the eight-element kernel's size (131,072 elements) and columns off its multiple."""
+    """Either side of the eight-element kernel's size (1,310,720 elements), with and without route weights, columns
+    off its multiple and the most rows in a workgroup (256)."""
     import ds41_gfx950 as G
     rng = np.random.default_rng(rows * cols)
     g, u = (O.bf16_bits((rng.standard_normal((rows, cols)) * 6).astype(np.float32)) for _ in range(2))
