@@ -66,11 +66,11 @@ def test_prefill_raw_vs_oracle(gpu, m, n, k):
     assert np.mean(got == ref) > 0.97
 
 
-@pytest.mark.parametrize("m", [15, 16, 17, 32, 33, 64, 81])
+@pytest.mark.parametrize("m", [15, 16, 17, 32, 33, 48, 49, 64, 81])
 @pytest.mark.parametrize("n,k,shift", [(136, 224, 0), (130, 256, 8), (257, 288, 3), (127, 1056, 2), (127, 1312, 1), (130, 2048, 1),
                                        (129, 2880, 1), (129, 32, 3), (129, 96, 1), (129, 128, 2), (129, 160, 1)])
 def test_prefill_raw_tile_edges(gpu, m, n, k, shift):
-    """Row blocks of 16, 32 and 64; channels past a 128-channel tile; k below, at and past one 256-k slice;
+    """Row blocks of 16, 32, 48 and 64; channels past a 128-channel tile; k below, at and past one 256-k slice;
     slices that end a round of three (1, 2, 6, 12), leave one (1) and leave two after whole rounds (5, 8), the last
     one whole or in part; rows of 1 to 5, 33 and 90 scale bytes; weights and scales at any byte offset.
     Each bf16 output rounds a sum of k products once; fp32 sums of up to 90 group dots differ by a few ulp,
