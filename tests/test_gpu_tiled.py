@@ -96,6 +96,11 @@ def test_tiled_layer_bitexact_down_rows(gpu, I):
     test_tiled_layer_bitexact(gpu, 8, 1024, I, 64, 8, True, False)
 
 
+@pytest.mark.parametrize("T,I", [(1, 256), (2, 1408), (3, 2304), (4, 2880), (2, 32)])
+def test_tiled_layer_bitexact_fused_down_rows(gpu, T, I):
+    """The same in the fused down + reduce kernel: rows of whole lines (256 and 2,304 channels), of part of one
+    (32), and whole and part (1,408 and 2,880)."""
+    test_tiled_layer_bitexact(gpu, T, 1024, I, 64, 4, True, False)
 
 def test_tiled_stack_with_host_tier_and_cache_bitexact(gpu):
     """A 3-layer stack at configs[4]'s layer shape (16 host-tier experts per layer) in both layouts: the tiled
