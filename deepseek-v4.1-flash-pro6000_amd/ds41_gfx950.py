@@ -190,7 +190,8 @@ def lib():
             ret, args = sig.split(":")
             for name in names.split():
                 f = getattr(L, "ds41_" + name)
-                f.restype, f.argtypes = _CTYPES[ret], [_CTYPES[a] for a in args]
+                # a char * argument may be bytes, a buffer, byref of one or an address: c_void_p takes all of them
+                f.restype, f.argtypes = _CTYPES[ret], [_CTYPES["p" if a == "s" else a] for a in args]
         _lib = L
     return _lib
 

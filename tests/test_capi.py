@@ -60,6 +60,20 @@ def test_binding_declares_every_entry_point():
     assert all(getattr(G.lib(), n).argtypes is not None for n in want)
 
 
+def test_binding_takes_any_error_buffer():
+    """An error buffer as an array, byref of it, a void pointer or its address, and a path as bytes or a char pointer."""
+    import ctypes
+    import sys
+    sys.path.insert(0, os.path.join(ROOT, "deepseek-v4.1-flash-pro6000_amd"))
+    import ds41_gfx950 as G
+    handle, path = ctypes.c_void_p(), b"/nonexistent/manifest"
+    for make in (lambda b: b, ctypes.byref, ctypes.addressof, lambda b: ctypes.cast(b, ctypes.c_void_p),
+                 lambda b: ctypes.c_void_p(ctypes.addressof(b)), lambda b: ctypes.cast(b, ctypes.c_char_p)):
+        for p in (path, ctypes.c_char_p(path)):
+            buf = ctypes.create_string_buffer(256)
+            assert G.lib().ds41_records_load(p, ctypes.byref(handle), make(buf), 256) == -1 and path in buf.value
+
+
 def test_abi_struct_sizes():
     import sys
     sys.path.insert(0, os.path.join(ROOT, "deepseek-v4.1-flash-pro6000_amd"))
