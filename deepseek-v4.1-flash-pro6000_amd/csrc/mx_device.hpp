@@ -605,17 +605,6 @@ __device__ __forceinline__ v4f mfma_chunk(const uint4 &lo, const uint4 &hi, cons
   const v8i a = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, bv, acc, 0, 4, 0, sa, 0, sw);
 }
-// The same chunk as two operands: its bytes with |v| >= 1 and its bytes with |v| < 1.
-__device__ __forceinline__ void split_chunk(const uint4 &lo, const uint4 &hi, v8i &big, v8i &small) {
-  const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t m = e4m3_big_mask(w[i]);
-    big[i] = (int)(w[i] & m);
-    small[i] = (int)(w[i] & ~m);
-  }
-}
-
 
 // Tiled weights (ds41_expert_slab_tile): the 16-byte K32 pieces of an MXFP4
 // matrix [N][K/2] stored in the MFMA B-operand order, piece (row n, group g) at
