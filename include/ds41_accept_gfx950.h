@@ -33,7 +33,7 @@ size_t ds41_spark_accept_workspace_bytes(int drafts, int vocab);
  * sampler's: a decision whose margin is within the bound on the difference
  * between parallel and sequential fp64 sums is recomputed with sequential sums.
  * flags bit 0 forces that sequential path for every decision (testing).
- * top_p < 1 with T > 0 returns hipErrorNotSupported in this version. */
+ * top_p < 1 with T > 0 keeps the host's nucleus (ds41_spark_probabilities) of every row. */
 int ds41_spark_verify_logits_gpu_v2(const float *target_logits, const float *draft_logits,
                                     const int32_t *drafts_dev, int drafts, int vocab,
                                     double temperature, double top_p, uint64_t seed, uint64_t step,

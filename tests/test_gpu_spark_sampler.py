@@ -244,7 +244,7 @@ def test_verify_gpu_v2_invalid_inputs_match_oracle(gpu):
         want = O.verify_gpu_v2(dd, qq, pp, 2, V, 0, 1, 2).raw()
         assert run_gpu(gpu, dd, qq, pp, 0, 1, 2) == want
         assert want[1] == -1
-    # an invalid row past the step's end is never read: the step is valid
+    # an invalid row past the step's end takes no part in it (its entries may be read): the step is valid
     late = p.copy(); late[2, 9] = np.nan
     want = O.verify_gpu_v2(np.array([0, 1], np.int32), q, late, 2, V, 0, 1, 2).raw()
     assert run_gpu(gpu, np.array([0, 1], np.int32), q, late, 0, 1, 2) == want
